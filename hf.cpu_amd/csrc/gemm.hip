@@ -32,7 +32,8 @@ extern "C" int hfa_gemm(const void* a, int a_dtype, int lda, const void* w, int 
         return rc ? rc : hfa_activation(out, ldo, out, ldo, out_dtype, M, N, act, stream);
     }
     HFA_REQUIRE(epilogue == 0, "gemm: the gate/up epilogue exists only on the matrix-core path");
-    const int rc = gemm_generic_launch(g);
+    const int rc = !force_plain && gemm_f32_supports(g) ? gemm_f32_launch(g, workspace, workspace_bytes, defer, pending_splits)
+                                                        : gemm_generic_launch(g);
     if (rc || !act) return rc;
     return hfa_activation(out, ldo, out, ldo, out_dtype, M, N, act, stream);
 }

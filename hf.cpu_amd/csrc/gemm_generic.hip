@@ -1,6 +1,6 @@
 // The plain matrix product: out[m, n] (+)= sum_k a[m, k] * w[n, k] + bias[n] with fp32
-// fused multiply-add in ascending k for every output element, whatever M is. It serves the
-// 32-bit path (no reduced-precision matrix mode) and every shape the MFMA kernels refuse.
+// fused multiply-add in ascending k for every output element, whatever M is. It serves every
+// mix of types and every shape that the matrix-core kernels (gemm_f32.hip, gemm_mfma.hip) refuse.
 // 64x64 or 128x128 output tile per 256-thread block, K in steps of 16 through LDS, 4x4 or 8x8 outputs a
 // thread; few rows have a kernel of their own further down.
 #include "common.h"

@@ -18,6 +18,11 @@ struct GemmArgs {
 // Any dtype mix, any size: fp32 multiply-add over K in ascending order for every output.
 int gemm_generic_launch(const GemmArgs& g);
 
+// fp32 x fp32 -> fp32 on the matrix cores (K and both row strides multiples of 4, 16-byte aligned bases), in an order of sums that K alone
+// sets. With `defer`, a product whose K was cut leaves its partial sums as below.
+bool gemm_f32_supports(const GemmArgs& g);
+int gemm_f32_launch(const GemmArgs& g, void* workspace, size_t workspace_bytes, int defer, int* pending_splits);
+
 // bf16 x bf16 on the matrix cores (K and both row strides multiples of 8, 16-byte aligned bases).
 // `workspace` holds the partial sums when K is split for small M; without one K is not split.
 // With `defer`, a product whose K was split leaves its partial sums in the workspace

@@ -469,14 +469,15 @@ __global__ __launch_bounds__(WM* WN* WAVE) void gemm_dma_kernel(
     }
 }
 
-// Sum of the K splits in ascending order, then bias and the output mode.
+// Sum of the K splits in ascending order (an accumulated output: onto its old value, as the norm adds the planes that a product
+// left to it), then bias and the output mode.
 template <int MODE>
 __global__ void gemm_finish_kernel(const float* __restrict__ partial, int splits, const float* __restrict__ bias,
                                    void* __restrict__ out, int ldo, int M, int N, int act) {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (size_t)M * N) return;
     const int row = (int)(idx / N), col = (int)(idx % N);
-    float v = 0.f;
+    float v = MODE == OUT_ACC ? reinterpret_cast<float*>(out)[(size_t)row * ldo + col] : 0.f;
     for (int s = 0; s < splits; s++) v += partial[(size_t)s * M * N + idx];
     if (bias) v += bias[col];
     if (MODE == OUT_BF16_ACT) v = hfa_act_apply(act, v);
@@ -488,10 +489,8 @@ __global__ void gemm_finish_kernel(const float* __restrict__ partial, int splits
             bf16_bits(hfa_gate_half(act, v) * up);
     } else if (IS_BF16_OUT(MODE))
         reinterpret_cast<uint16_t*>(out)[(size_t)row * ldo + col] = bf16_bits(v);
-    else if (MODE == OUT_F32)
-        reinterpret_cast<float*>(out)[(size_t)row * ldo + col] = v;
     else
-        reinterpret_cast<float*>(out)[(size_t)row * ldo + col] += v;
+        reinterpret_cast<float*>(out)[(size_t)row * ldo + col] = v;
 }
 
 // The gate/up case of the above, four results a thread: 16-byte loads of every plane asked for
