@@ -302,6 +302,7 @@ extern "C" int hfa_paged_attention(const void* q, int dtype, int ldq, const void
         }
         return 0;
     }
+    if (!force_plain && !slopes && !cross_values && dtype == HFA_F32 && attn_f32_supports(a)) return attn_f32_launch(a);
     // one key/value head with wide keys and values of a size of their own, read by every query head
     if (!force_plain && !slopes && !cross_values && dtype == HFA_BF16 && attn_shared_supports(a, v_head_dim, v_width))
         return attn_shared_launch(a, v_head_dim);

@@ -81,6 +81,10 @@ inline bool attn_masked_mode(const AttnArgs& a) {
 bool attn_masked_sizes(int head_dim, int v_head_dim);
 int attn_masked_run(const AttnArgs& a, const AttnCut& c);
 
+// 32 bits on the matrix cores: a softmax over a head's own values; see attention_f32.hip for what it needs.
+bool attn_f32_supports(const AttnArgs& a);
+int attn_f32_launch(const AttnArgs& a);
+
 // bf16 on the matrix cores; see attention_mfma.hip for what it needs.
 bool attn_mfma_supports(const AttnArgs& a);
 int attn_mfma_launch(const AttnArgs& a);
