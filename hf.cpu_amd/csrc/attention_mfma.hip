@@ -197,14 +197,24 @@ int attn_mfma_launch(const AttnArgs& a) {
     int span = a.window > 0 && a.window + a.max_q_len < a.max_seq_len ? a.window + a.max_q_len : a.max_seq_len;
     if (a.mask_chunk > 0 && a.mask_chunk + a.max_q_len < span) span = a.mask_chunk + a.max_q_len;      // a masking chunk bounds the keys as a window does
     int n_chunks = 1, chunk_keys = a.max_seq_len;
-    // How many waves in all is a measured choice. Head size 128 (7B shape): 512; with 1,024 a step took 1.3 % longer
-    // at 64 sequences and 4.5 % longer at 8 sequences of 16,384 tokens, with 256 more than that. Head size 64 (0.5B
-    // shape), where a wave has half the work per key: 1,024; with 512 a step of 64 sequences took 4.5 % longer; but no
-    // chunk of fewer than 128 keys for either head size (with chunks of 64 keys a step of 8 sequences of the 0.5B shape at
-    // 2,048 took 5 % longer, one of 16 2 %; one of 2 sequences of the 7B shape 2 % longer).
+    // How many waves in all is a measured choice. At least 512 with head size 128 (8 sequences of 16,384 tokens, 7B shape: 4.83 ms a
+    // step; with 1,024 waves 4.96) and 1,024 with head size 64, where a wave has half the work per key (64 sequences of the 0.5B
+    // shape: 512 take 4.5 % longer); but no chunk of fewer than 128 keys (with chunks of 64 a step of 8 sequences of the 0.5B shape at
+    // 2,048 took 5 % longer, one of 2 sequences of the 7B shape 2 %).
+    // Up to 4,096 keys and 512 columns' tiles more chunks than that: about 224 keys each, up to 16 chunks and 2,048 waves. Requests
+    // of a batch differ in length, and a long one's chunk outlasts all the others (a step of the 7B shape with 64 requests of 64 to
+    // 2,048 tokens: 2 chunks 5.72 ms, 4 5.54, 8 5.35; with 128 of up to 1,500: 1 chunk 7.08, 4 6.42; of the 3B shape with 40 of up
+    // to 2,000: 7 chunks 3.46, 10 3.35); where all are long it costs nothing (64 of 2,020: 6.09 against 6.04 ms). Beyond 4,096 keys it does (48 of
+    // 16,000: 3 chunks 12.6 ms, 8 13.0), and from 200 requests on the batch fills the machine by itself (700 keys: 1 chunk 8.36, 4 8.55).
     const int fill = a.head_dim > 64 ? 512 : 1024;
-    if (waves < fill && span > 128 && a.workspace) {
-        int want = (int)((fill + waves - 1) / waves);
+    int want = (int)((fill + waves - 1) / waves);
+    if (waves <= 512 && span <= 4096) {
+        int more = (span + 223) / 224;
+        if (more > 16) more = 16;
+        if (more > 2048 / waves) more = (int)(2048 / waves);
+        if (want < more) want = more;
+    }
+    if (want > 1 && span > 128 && a.workspace) {
         const int most = (span + 127) / 128;
         if (want > most) want = most;
         // under a window or a mask by chunks the cuts are counted from the tile's first key block: they cover what a tile can see
