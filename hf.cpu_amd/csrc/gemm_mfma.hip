@@ -629,6 +629,74 @@ int gemm_mode_of(const GemmArgs& g) {
     return g.accumulate ? OUT_ACC : (g.out_dtype == HFA_BF16 ? (g.act ? OUT_BF16_ACT : OUT_BF16) : OUT_F32);
 }
 
+// ---- which tiles, and how many parts of K, for more than 128 rows ----
+//
+// A tile kind's time for a product, as measured over 5,000 (sizes, kind, parts) at 70 to 2,048 rows of the q/k/v, o, gate+up and down
+// products of the 0.5B, 1.5B, 3B and 7B shapes (median error of the formula 5 to 10 %): blocks go over the CUs in rounds; a block
+// multiplies at `rate` TFLOP/s, or at its share of `cap` (all CUs together: the power and the caches' bandwidth set that), and costs
+// `round` us beside it (negative where two blocks share a CU: one starts while the other multiplies); `start` us once. Results that
+// are added to an fp32 output cost `acc` us a MB read and written, planes of partial sums `part` us a MB.
+struct TileKind {
+    int bm, bn, per_cu;
+    double rate, cap, round, start, acc, part;
+};
+enum { TILE_256x256, TILE_256x192, TILE_256x128, TILE_128x128, TILE_128x128_REG, TILE_KINDS };
+static const TileKind tile_kinds[TILE_KINDS] = {
+    {256, 256, 1, 6.45, 1196., 5.7, 3.6, 0.95, 0.132},
+    {256, 192, 1, 5.86, 1184., 3.3, 4.8, 0.84, 0.154},
+    {256, 128, 1, 4.90, 980., 2.3, 5.0, 0.68, 0.135},
+    {128, 128, 2, 3.66, 845., -0.8, 8.8, 0.67, 0.145},
+    {128, 128, 2, 3.44, 1067., -1.2, 8.8, 0.40, 0.131},
+};
+struct TileChoice {
+    int kind, parts, part_k;
+    double us;
+};
+
+// Microseconds of the product with `parts` parts of K, and of what the planes cost whoever adds them up: the norm that reads them
+// anyway (5 TB/s), the rotation and store (4 TB/s, and a slower kernel than the one for finished rows) or a finishing kernel.
+static double tile_us(const GemmArgs& g, int mode, int kind, int parts, bool defer) {
+    const TileKind& t = tile_kinds[kind];
+    const long blocks = (long)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn) * parts;
+    const int steps = ((g.K + parts - 1) / parts + 31) / 32;
+    const double work = (double)t.bm * t.bn * 64 * steps / 1e6, mb = (double)g.M * g.N * 4 / 1e6;
+    auto round_us = [&](long b) { return work / (t.rate < t.cap / b ? t.rate : t.cap / b) + t.round; };
+    double us = t.start + blocks / 256 * round_us(256) + (blocks % 256 ? round_us(blocks % 256) : 0.0);
+    if (parts > 1) us += parts * mb * t.part;
+    else if (mode == OUT_ACC) us += 2 * mb * t.acc;
+    const double weights_us = (double)g.N * g.K * 2 / 4.6e6 + 5;
+    if (us < weights_us) us = weights_us;
+    if (parts > 1) us += 2 + (mode == OUT_ACC ? parts * mb / 5.0 : parts * mb / 4.0 + 2) + (defer ? 0 : 5);
+    return us;
+}
+
+// Another kind or number of parts than `now` if the formula gives it 6 % less time (closer calls it does not tell apart). Gate and up
+// columns meet inside a block, which rules out parts and tiles of 192; `rows_ok` and `dma_ok`: operands (and 16-bit results) that the
+// kernels of direct loads take. What it changes, measured: down of the 7B shape at 333 rows 103 us to 80 (three parts of 128 x 128 tiles, or six of
+// 256 x 128, where four parts of the register-staged tiles were taken), o at 512 rows 36 to 26 (two parts, not seven), down of the
+// 0.5B shape at 2,048 rows 48 to 32 (two parts of 128 x 128, not eight of 256 x 256), its gate+up 63 to 52 (304 tiles of 256 x 256 are two
+// rounds of which the second is nearly empty).
+static TileChoice better_tiles(const GemmArgs& g, int mode, TileChoice now, bool rows_ok, bool dma_ok, size_t workspace_bytes, bool defer) {
+    now.us = tile_us(g, mode, now.kind, now.parts, defer);
+    TileChoice best = now;
+    for (int kind = 0; kind < TILE_KINDS; kind++) {
+        const TileKind& t = tile_kinds[kind];
+        const bool staged = kind == TILE_128x128_REG;
+        const long tiles = (long)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
+        if ((!staged && !rows_ok) || (mode == OUT_SWIGLU && kind == TILE_256x192)) continue;
+        for (int parts = 1; parts <= 12; parts++) {
+            if (parts == 1 && !staged && !dma_ok) continue;
+            if (parts > 1 && (mode == OUT_SWIGLU || g.K / parts < 256 || tiles * parts > 550 * t.per_cu ||
+                              (size_t)parts * g.M * g.N * sizeof(float) > workspace_bytes))
+                break;
+            const int unit = staged ? 64 : 32, part_k = ((g.K + unit - 1) / unit + parts - 1) / parts * unit;
+            const TileChoice c = {kind, (g.K + part_k - 1) / part_k, part_k, tile_us(g, mode, kind, parts, defer)};
+            if (c.us < 0.94 * now.us && c.us < best.us) best = c;
+        }
+    }
+    return best;
+}
+
 int gemm_mfma_launch(const GemmArgs& g, void* workspace, size_t workspace_bytes, int defer, int* pending_splits) {
     const int mode = gemm_mode_of(g);
     if (pending_splits) *pending_splits = 0;
@@ -679,16 +747,13 @@ int gemm_mfma_launch(const GemmArgs& g, void* workspace, size_t workspace_bytes,
     }
     int k_per_split = ((k_tiles + splits - 1) / splits) * BK;
     splits = (g.K + k_per_split - 1) / k_per_split;
-    const int kmode = splits > 1 ? OUT_PARTIAL : mode;
-    void* kout = splits > 1 ? workspace : g.out;
-    int rc;
     // Long prompts: tiles of 256 rows fed by direct loads into LDS, if the rows they waste past M
     // cost less than they gain (they run about a quarter faster than the 128 x 128 tiles).
     const int rows256 = (g.M + 255) / 256 * 256, rows128 = (g.M + 127) / 128 * 128;
-    const bool rows_ok = BM == 128 && g.K % 64 == 0 && g.lda < (1 << 22) && g.ldw < (1 << 22) &&
-                         (size_t)rows256 * 100 <= (size_t)rows128 * 128;
-    const bool dma_ok = rows_ok && splits == 1 &&
-                        (g.out_dtype != HFA_BF16 || (g.ldo % 8 == 0 && g.N % 16 == 0 && ((uintptr_t)g.out & 15) == 0));
+    const bool direct_ok = BM == 128 && g.K % 64 == 0 && g.lda < (1 << 22) && g.ldw < (1 << 22);
+    const bool out_ok = g.out_dtype != HFA_BF16 || (g.ldo % 8 == 0 && g.N % 16 == 0 && ((uintptr_t)g.out & 15) == 0);
+    const bool rows_ok = direct_ok && (size_t)rows256 * 100 <= (size_t)rows128 * 128;
+    const bool dma_ok = rows_ok && splits == 1 && out_ok;
     const int tiles256 = (rows256 / 256) * ((g.N + 255) / 256);
     // A narrow output has too few 256 x 256 tiles for the CUs: K is cut into as many parts as give
     // every CU a block (at most one round of blocks, parts of 512 columns at least) and the parts' sums
@@ -738,31 +803,38 @@ int gemm_mfma_launch(const GemmArgs& g, void* workspace, size_t workspace_bytes,
     const int tiles192 = (rows256 / 256) * ((g.N + 191) / 192);
     const bool narrow = dma_ok && tiles256 >= 128 && mode != OUT_SWIGLU &&
                         ((tiles192 + cus - 1) / cus) * 80 < ((tiles256 + cus - 1) / cus) * 100;
-    if (narrow)
-        rc = launch_dma<256, 192, 32, 4, 2, 5>(g, kmode, kout, 1, g.K);
-    else if (dma_ok && tiles256 >= 128)
-        rc = launch_dma<256, 256, 32, 2, 4, 4>(g, kmode, kout, 1, g.K);
-    else if (halves) {
-        rc = half_wide ? launch_dma<256, 128, 32, 4, 2, 6>(g, OUT_PARTIAL, workspace, parts, part_k)
-                       : launch_dma<256, 256, 32, 2, 4, 4>(g, OUT_PARTIAL, workspace, parts, part_k);
-        if (rc) return rc;
-        if (defer && pending_splits) {
-            *pending_splits = parts;
-            return 0;
+    int rc;
+    if (BM == 128) {
+        TileChoice c = {TILE_128x128_REG, splits, k_per_split, 0};
+        if (narrow) c = {TILE_256x192, 1, g.K, 0};
+        else if (dma_ok && tiles256 >= 128) c = {TILE_256x256, 1, g.K, 0};
+        else if (halves) c = {half_wide ? TILE_256x128 : TILE_256x256, parts, part_k, 0};
+        else if (dma_ok && 2 * tiles256 >= 128) c = {TILE_256x128, 1, g.K, 0};
+        if (g.M > 128) c = better_tiles(g, mode, c, direct_ok, direct_ok && out_ok, workspace ? workspace_bytes : 0, defer);
+        splits = c.parts;
+        k_per_split = c.part_k;
+        const int kmode = splits > 1 ? OUT_PARTIAL : mode;
+        void* kout = splits > 1 ? workspace : g.out;
+        switch (c.kind) {
+            case TILE_256x256: rc = launch_dma<256, 256, 32, 2, 4, 4>(g, kmode, kout, splits, k_per_split); break;
+            case TILE_256x192: rc = launch_dma<256, 192, 32, 4, 2, 5>(g, kmode, kout, splits, k_per_split); break;
+            case TILE_256x128: rc = launch_dma<256, 128, 32, 4, 2, 6>(g, kmode, kout, splits, k_per_split); break;
+            case TILE_128x128: rc = launch_dma<128, 128, 32, 2, 2, 5>(g, kmode, kout, splits, k_per_split); break;
+            // eight waves a block: about 2 % quicker than four with twice the accumulators
+            default: rc = launch_mode<128, 128, 64, 4, 2>(g, kmode, kout, splits, k_per_split);
         }
-        return gemm_finish_launch((const float*)workspace, parts, g.bias, g.out, mode, g.ldo, g.M, g.N, g.stream, g.act);
-    } else if (dma_ok && 2 * tiles256 >= 128)
-        rc = launch_dma<256, 128, 32, 4, 2, 6>(g, kmode, kout, 1, g.K);
-    else if (BM == 128)                        // eight waves a block in both: about 2 % quicker than four with twice the accumulators
-        rc = launch_mode<128, 128, 64, 4, 2>(g, kmode, kout, splits, k_per_split);
-    else if (BM == 64 && kmode == OUT_SWIGLU)  // a wave needs 64 columns to pair gate and up
-        rc = launch_mode<64, 128, 64, 2, 2>(g, kmode, kout, splits, k_per_split);
-    else if (BM == 64)
-        rc = launch_mode<64, 128, 64, 2, 4>(g, kmode, kout, splits, k_per_split);
-    else if (kmode == OUT_SWIGLU)
-        rc = launch_mode<32, 128, 64, 1, 2>(g, kmode, kout, splits, k_per_split);
-    else
-        rc = launch_mode<32, 128, 64, 1, 4>(g, kmode, kout, splits, k_per_split);
+    } else {
+        const int kmode = splits > 1 ? OUT_PARTIAL : mode;
+        void* kout = splits > 1 ? workspace : g.out;
+        if (BM == 64 && kmode == OUT_SWIGLU)       // a wave needs 64 columns to pair gate and up
+            rc = launch_mode<64, 128, 64, 2, 2>(g, kmode, kout, splits, k_per_split);
+        else if (BM == 64)
+            rc = launch_mode<64, 128, 64, 2, 4>(g, kmode, kout, splits, k_per_split);
+        else if (kmode == OUT_SWIGLU)
+            rc = launch_mode<32, 128, 64, 1, 2>(g, kmode, kout, splits, k_per_split);
+        else
+            rc = launch_mode<32, 128, 64, 1, 4>(g, kmode, kout, splits, k_per_split);
+    }
     if (rc || splits == 1) return rc;
     if (defer && pending_splits) {             // the caller sums the partial results in its next kernel
         *pending_splits = splits;
