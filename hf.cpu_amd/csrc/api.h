@@ -368,6 +368,12 @@ int hfa_draw_rows(float* vals, const int* ids, int n_rows, int vocab, const floa
 int hfa_topk(const float* logits, int ld, int* ids, float* vals, float* stats, int n_rows, int vocab, int k,
              hipStream_t stream);
 
+// The same without stats, with a workspace of hfa_topk_cut_workspace(n_rows, vocab) bytes (8-byte aligned): rows are cut into slices that
+// spread over the machine where k and the vocabulary allow it; without enough workspace it is hfa_topk.
+size_t hfa_topk_cut_workspace(int n_rows, int vocab);
+int hfa_topk_cut(const float* logits, int ld, int* ids, float* vals, int n_rows, int vocab, int k, void* workspace, size_t workspace_bytes,
+                 hipStream_t stream);
+
 // Random weights on the device: element e of the tensor with `key` by the counter-based rule that
 // weights/random_init.py states (the host's writer computes the same bits). dtype HFA_F32 or HFA_BF16
 // with rule 0 (N(0, std): scale = std / sqrt(8 (65536^2 - 1) / 12)) or 1 (1 + that); dtype 2 (int32)

@@ -235,9 +235,8 @@ __device__ void topk_sort_and_store(float* cand_v, int* cand_i, int found, int k
     }
 }
 
-__global__ __launch_bounds__(TOPK_THREADS) void topk_kernel(const float* __restrict__ logits, int ld,
-                                                            int* __restrict__ ids, float* __restrict__ vals,
-                                                            float* __restrict__ stats, int vocab, int k) {
+__device__ void topk_row(const float* __restrict__ logits, int ld, int* __restrict__ ids, float* __restrict__ vals, float* __restrict__ stats,
+                         int vocab, int k) {
     __shared__ uint32_t hist[2048];
     __shared__ float cand_v[TOPK_MAX];
     __shared__ int cand_i[TOPK_MAX];
@@ -382,6 +381,194 @@ __global__ __launch_bounds__(TOPK_THREADS) void topk_kernel(const float* __restr
     }
     __syncthreads();
     topk_sort_and_store(cand_v, cand_i, k, k, ids, vals);
+}
+
+__global__ __launch_bounds__(TOPK_THREADS) void topk_kernel(const float* __restrict__ logits, int ld,
+                                                            int* __restrict__ ids, float* __restrict__ vals,
+                                                            float* __restrict__ stats, int vocab, int k) {
+    topk_row(logits, ld, ids, vals, stats, vocab, k);
+}
+
+// The best k of rows without their log-sum-exp, in two launches: one block a row (above) reads a row twice at what one CU's loads give,
+// which for 64 rows of 151,936 is 60 us on a quarter of the CUs. Here a row is cut into slices of up to PART_THREADS x PART_EACH logits,
+// a block each (960 blocks for those rows), read once into registers. As above, the k-th largest of the threads' own maxima is a bound that the
+// row's k-th largest reaches; a slice leaves what reaches its bound. The second launch keeps, a block a row, what reaches the largest of the
+// slices' bounds, in LDS, and gives each its place by counting the better ones in sorted lists of 64 (the same place whatever order they came in).
+// Rows that leave too much (ties by the hundred) or too little (NaNs) go the way above. With k 40: 21 us for those rows (58), 17 us
+// for one of them (52).
+#define PART_THREADS 512
+#define PART_EACH 20
+#define PART_KEEP 512                                        // candidates a slice may leave
+#define PART_MOST_K 256
+#define ROW_KEEP 2048                                        // candidates of a row in LDS
+
+struct PartHead {
+    int found;                                               // may exceed PART_KEEP: then not all of them were left
+    float bound;
+};
+
+__global__ __launch_bounds__(PART_THREADS) void topk_part_kernel(const float* __restrict__ logits, int ld, int vocab, int k,
+                                                                 PartHead* __restrict__ heads, float2* __restrict__ left) {
+    __shared__ float sorted[PART_THREADS / WAVE][WAVE];
+    __shared__ float bound;
+    __shared__ int found;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE, parts = gridDim.y;
+    const int per = (vocab + parts - 1) / parts, lo = blockIdx.y * per, hi = lo + per < vocab ? lo + per : vocab;
+    const float* row = logits + (size_t)blockIdx.x * ld;
+    float v[PART_EACH], top = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < PART_EACH; u++) {
+        const int i = lo + u * PART_THREADS + tid;
+        v[u] = row[i < hi ? i : lo];                         // (no condition around a load: they all travel together)
+    }
+#pragma unroll
+    for (int u = 0; u < PART_EACH; u++) {
+        if (lo + u * PART_THREADS + tid >= hi) v[u] = -INFINITY;
+        top = fmaxf(top, v[u]);
+    }
+    if (tid == 0) found = 0;
+    // the wave's 64 maxima in descending order, by a bitonic network across its lanes
+    float x = top;
+#pragma unroll
+    for (int size = 2; size <= WAVE; size <<= 1)
+#pragma unroll
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+            const float y = __shfl_xor(x, stride, WAVE);
+            const bool high = ((lane & stride) == 0) == ((lane & size) == 0);      // this lane keeps the larger of the two
+            x = high ? fmaxf(x, y) : fminf(x, y);
+        }
+    sorted[wave][lane] = x;
+    __syncthreads();
+    // its place among all maxima: in its own list, and the number of larger ones (of equal ones: in earlier lists) in the others
+    int rank = lane;
+    for (int w = 0; w < PART_THREADS / WAVE; w++) {
+        if (w == wave) continue;
+        int n = 0;                                           // entries of list w that come before x
+#pragma unroll
+        for (int step = WAVE / 2; step > 0; step >>= 1) {
+            const float y = sorted[w][n + step - 1];
+            if (y > x || (y == x && w < wave)) n += step;
+        }
+        const float y = sorted[w][n];
+        rank += n + ((y > x || (y == x && w < wave)) ? 1 : 0);
+    }
+    if (rank == k - 1) bound = x;
+    __syncthreads();
+    const float least = bound;
+    const size_t slice = (size_t)blockIdx.x * parts + blockIdx.y;
+    float2* mine = left + slice * PART_KEEP;
+#pragma unroll
+    for (int u = 0; u < PART_EACH; u++) {
+        const int i = lo + u * PART_THREADS + tid;
+        if (i < hi && v[u] >= least) {
+            const int at = atomicAdd(&found, 1);
+            if (at < PART_KEEP) mine[at] = make_float2(v[u], __int_as_float(i));
+        }
+    }
+    __syncthreads();
+    if (tid == 0) heads[slice] = PartHead{found, least};
+}
+
+// Larger logit <=> larger upper half; of equal ones the smaller id <=> the larger lower half. No candidate's key is 0.
+__device__ __forceinline__ unsigned long long candidate_key(float v, int i) {
+    return ((unsigned long long)float_key(v) << 32) | (0xffffffffu - (uint32_t)i);
+}
+
+__global__ __launch_bounds__(TOPK_THREADS) void topk_join_kernel(const float* __restrict__ logits, int ld, int* __restrict__ ids,
+                                                                 float* __restrict__ vals, int vocab, int k, int parts,
+                                                                 const PartHead* __restrict__ heads, const float2* __restrict__ left) {
+    __shared__ unsigned long long cand[ROW_KEEP];
+    __shared__ int n_cand;
+    __shared__ float red[17];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
+    const PartHead* head = heads + (size_t)blockIdx.x * parts;
+    float least = -INFINITY;
+    bool whole = true;
+    for (int p = tid; p < parts; p += TOPK_THREADS) {
+        least = fmaxf(least, head[p].bound);
+        whole = whole && head[p].found <= PART_KEEP;
+    }
+    if (tid == 0) n_cand = 0;
+    least = block_max(least, red);
+    whole = __syncthreads_and(whole);
+    if (whole) {
+        for (int p = wave; p < parts; p += TOPK_THREADS / WAVE) {
+            const int found = head[p].found;
+            for (int c = lane; c < found; c += WAVE) {
+                const float2 x = left[((size_t)blockIdx.x * parts + p) * PART_KEEP + c];
+                if (x.x >= least) {
+                    const int at = atomicAdd(&n_cand, 1);
+                    if (at < ROW_KEEP) cand[at] = candidate_key(x.x, __float_as_int(x.y));
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const int n = n_cand;
+    if (!whole || n < k || n > ROW_KEEP) {                   // (uniform)
+        topk_row(logits, ld, ids, vals, nullptr, vocab, k);
+        return;
+    }
+    // lists of 64 in descending order, a wave each
+    const int lists = (n + WAVE - 1) / WAVE;
+    for (int l = wave; l < lists; l += TOPK_THREADS / WAVE) {
+        unsigned long long x = l * WAVE + lane < n ? cand[l * WAVE + lane] : 0;
+#pragma unroll
+        for (int size = 2; size <= WAVE; size <<= 1)
+#pragma unroll
+            for (int stride = size >> 1; stride > 0; stride >>= 1) {
+                const unsigned long long y = __shfl_xor(x, stride, WAVE);
+                const bool high = ((lane & stride) == 0) == ((lane & size) == 0);
+                x = (x > y) == high ? x : y;
+            }
+        cand[l * WAVE + lane] = x;
+    }
+    __syncthreads();
+    // a candidate's place: the better ones in its own list and in each of the others
+    for (int l = wave; l < lists; l += TOPK_THREADS / WAVE) {
+        const unsigned long long x = cand[l * WAVE + lane];
+        int place = lane;
+        for (int o = 0; o < lists; o++) {
+            const unsigned long long* list = cand + o * WAVE;
+            int better_ones = 0;
+#pragma unroll
+            for (int step = WAVE / 2; step > 0; step >>= 1)
+                if (list[better_ones + step - 1] > x) better_ones += step;
+            better_ones += list[better_ones] > x;
+            place += o == l ? 0 : better_ones;
+        }
+        if (x != 0 && place < k) {
+            const int i = (int)(0xffffffffu - (uint32_t)x);
+            ids[(size_t)blockIdx.x * k + place] = i;
+            vals[(size_t)blockIdx.x * k + place] = logits[(size_t)blockIdx.x * ld + i];
+        }
+    }
+}
+
+static int topk_parts(int vocab) { return (vocab + PART_THREADS * PART_EACH - 1) / (PART_THREADS * PART_EACH); }
+
+extern "C" size_t hfa_topk_cut_workspace(int n_rows, int vocab) {
+    return (size_t)n_rows * topk_parts(vocab) * (sizeof(PartHead) + PART_KEEP * sizeof(float2));
+}
+
+extern "C" int hfa_topk_cut(const float* logits, int ld, int* ids, float* vals, int n_rows, int vocab, int k, void* workspace,
+                            size_t workspace_bytes, hipStream_t stream) {
+    HFA_REQUIRE(n_rows > 0 && vocab > 0 && ld >= vocab, "topk: bad sizes rows=%d vocab=%d ld=%d", n_rows, vocab, ld);
+    HFA_REQUIRE(k >= 0 && k <= 1024 && k <= vocab, "topk: k=%d is outside 0..min(1024, vocab)", k);
+    HFA_REQUIRE(k == 0 || (ids && vals), "topk: no output for the candidates");
+    // two slices at least (a row of one is read at once by the kernel above), k among a slice's maxima with room to spare, and no more
+    // candidates than the second launch holds (every slice leaves about k; 15 slices with k 200 went the long way at last: 80 us against 62)
+    const int parts = topk_parts(vocab);
+    if (parts < 2 || parts > 65535 || k < 1 || k > PART_MOST_K || (long)k * parts > ROW_KEEP || !workspace || ((uintptr_t)workspace & 7) != 0 ||
+        workspace_bytes < hfa_topk_cut_workspace(n_rows, vocab))
+        return hfa_topk(logits, ld, ids, vals, nullptr, n_rows, vocab, k, stream);
+    PartHead* heads = (PartHead*)workspace;
+    float2* left = (float2*)(heads + (size_t)n_rows * parts);
+    topk_part_kernel<<<dim3(n_rows, parts), PART_THREADS, 0, stream>>>(logits, ld, vocab, k, heads, left);
+    HFA_LAUNCH_CHECK("topk_part");
+    topk_join_kernel<<<n_rows, TOPK_THREADS, 0, stream>>>(logits, ld, ids, vals, vocab, k, parts, heads, left);
+    HFA_LAUNCH_CHECK("topk_join");
+    return 0;
 }
 
 extern "C" int hfa_topk(const float* logits, int ld, int* ids, float* vals, float* stats, int n_rows, int vocab,

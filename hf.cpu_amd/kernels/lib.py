@@ -62,6 +62,7 @@ _SIGNATURES = {
     "hfa_argmax": [P, I, P, I, I, P, c_size_t, P],
     "hfa_argmax_static": [P, I, P, I, I, P],
     "hfa_topk": [P, I, P, P, P, I, I, I, P],
+    "hfa_topk_cut": [P, I, P, P, I, I, I, P, c_size_t, P],
     "hfa_order_rows": [P, I, P, P, P, I, I, P, c_size_t, P],
     "hfa_draw_rows": [P, P, I, I, P, P, P, P],
     "hfa_random_fill": [P, I, c_size_t, ctypes.c_uint64, F, I, I, P],

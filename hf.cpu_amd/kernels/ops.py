@@ -1564,6 +1564,10 @@ class Ops:
         ids = memory.empty((R, max(k, 1)), torch.int32, logits.device, "top-k ids")
         vals = memory.empty((R, max(k, 1)), torch.float32, logits.device, "top-k values")
         stats = memory.empty((R, 2), torch.float32, logits.device, "row statistics") if want_stats else None
-        self._check(self.lib.hfa_topk(logits.data_ptr(), _rows(logits, "topk logits"), ids.data_ptr(), vals.data_ptr(),
-                                      None if stats is None else stats.data_ptr(), R, V, k, self._stream()))
+        if stats is None:
+            self._check(self.lib.hfa_topk_cut(logits.data_ptr(), _rows(logits, "topk logits"), ids.data_ptr(), vals.data_ptr(), R, V, k,
+                                              self.workspace.data_ptr(), self.workspace.numel(), self._stream()))
+        else:
+            self._check(self.lib.hfa_topk(logits.data_ptr(), _rows(logits, "topk logits"), ids.data_ptr(), vals.data_ptr(),
+                                          stats.data_ptr(), R, V, k, self._stream()))
         return ids[:, :k], vals[:, :k], stats
