@@ -20,6 +20,7 @@ import torch
 
 from .. import memory
 from ..status import EINVAL, fail
+from .rng import uniforms
 
 TOPK_KERNEL_MAX = 1024
 f32 = np.float32
@@ -137,26 +138,42 @@ class Sampler:
         R, V = logits.shape
         if R != len(wants):
             fail(EINVAL, f"sampler: {R} rows of logits for {len(wants)} requests")
-        if any(n_lp for _, _, n_lp in wants):
+        from_best = bool(R) and self._drawn_from_best(wants, V)
+        if not from_best and any(n_lp for _, _, n_lp in wants):
             return Started(None, self.sample(logits, wants))
-        if all(p.greedy for p, _, _ in wants):
+        if not from_best and all(p.greedy for p, _, _ in wants):
             arg = self.ops.argmax(logits)
             read = self._to_host_later(arg)
             return Started(arg, None, lambda: [Choice(int(t)) for t in read()])
-        if all(not p.greedy and 0 < p.top_k <= TOPK_KERNEL_MAX and p.top_k < V for p, _, _ in wants):
-            k = max(p.top_k for p, _, _ in wants)
-            ids, vals, _ = self.ops.topk(logits, k, want_stats=False)
-            numbers = np.array([(p.temp, p.top_p, p.min_p, rng.uniform()) for p, rng, _ in wants], dtype=f32)
-            cuts = np.array([p.top_k for p, _, _ in wants], dtype=np.int32)
-            drawn = self._draw(ids, vals, numbers, cuts, on_device=True)
+        if from_best:
+            drawn = self._draw_from_best(logits, wants)
             read = self._to_host_later(drawn)
-            return Started(drawn, None, lambda: [Choice(int(t)) for t in read()])
+            return Started(drawn, None, lambda: [Choice(t) for t in read().tolist()])
         return Started(None, self.sample(logits, wants))
+
+    @staticmethod
+    def _drawn_from_best(wants, vocab):
+        """Whether every row is drawn from its best k, without log-probabilities."""
+        return all(not n_lp and not p.greedy and 0 < p.top_k <= TOPK_KERNEL_MAX and p.top_k < vocab for p, _, n_lp in wants)
+
+    def _draw_from_best(self, logits, wants):
+        """The rows' tokens, on the device, where ``_drawn_from_best`` holds."""
+        cuts = np.array([p.top_k for p, _, _ in wants], dtype=np.int32)
+        ids, vals, _ = self.ops.topk(logits, int(cuts.max()), want_stats=False)
+        # the rows' numbers are put together while the device looks for their best
+        numbers = np.empty((len(wants), 4), dtype=f32)
+        numbers[:, 0] = [p.temp for p, _, _ in wants]
+        numbers[:, 1] = [p.top_p for p, _, _ in wants]
+        numbers[:, 2] = [p.min_p for p, _, _ in wants]
+        numbers[:, 3] = uniforms([rng for _, rng, _ in wants])
+        return self._draw(ids, vals, numbers, cuts, on_device=True)
 
     def sample(self, logits, wants):
         R = logits.shape[0]
         if R != len(wants):
             fail(EINVAL, f"sampler: {R} rows of logits for {len(wants)} requests")
+        if R and self._drawn_from_best(wants, logits.shape[1]):
+            return [Choice(t) for t in self._draw_from_best(logits, wants).cpu().tolist()]
         out = [None] * R
         need_k = 0
         for params, _, n_lp in wants:
@@ -168,7 +185,7 @@ class Sampler:
         arg = self.ops.argmax(logits).cpu().numpy() if greedy else None
         best = ids = vals = stats = None
         if need_k or any(n for _, _, n in wants):
-            best = self.ops.topk(logits, need_k)
+            best = self.ops.topk(logits, need_k, want_stats=any(n for _, _, n in wants))
             if any(n for _, _, n in wants):       # before the draw below turns the values into probabilities
                 ids, vals, stats = (t.cpu().numpy() for t in best)
         toks = [None] * R

@@ -114,3 +114,15 @@ def test_sticky_output_error():
     o.event("x")
     assert o.err
     o.event("y")
+
+
+def test_many_generators_at_once():
+    """``uniforms`` draws what each generator draws by itself, for few, for many and for one that stands twice."""
+    from hf_cpu_amd.sampling.rng import Rng, uniforms
+    for n in (1, 7, 8, 64):
+        a, b = [Rng(i * 977) for i in range(n)], [Rng(i * 977) for i in range(n)]
+        for _ in range(3):
+            assert list(uniforms(a)) == [r.uniform() for r in b]
+            assert [r.s for r in a] == [r.s for r in b] and all(type(r.s) is int for r in a)
+    one, same = Rng(5), Rng(5)
+    assert list(uniforms([one] * 9)) == [same.uniform() for _ in range(9)]
