@@ -221,7 +221,88 @@ extern "C" size_t hfa_linear_scan_state_floats(int n_heads, int qk_dim, int v_di
     return (size_t)n_heads * ns * npt * p_pad;
 }
 
-template <typename T, typename TS, int NS, int NPT>
+// A chunk's keys or queries (or what else has a value a key channel) on their way to LDS, raw: a conversion or a mask beside
+// the load would wait for it, and the loads of a chunk then make their trips to memory one after another (bf16: 33 trips
+// where one will do). WIDE: pieces of four values (rows, leading dimensions and the head's width allow it). Otherwise a value
+// a load. Measured with the places in LDS below, before and after, 16 heads of 128 x 128: exponential gates
+// on bf16, four requests of 357 to 900 tokens 399 and 252 us, sixteen of 300 tokens 583 and 256, single tokens of 64
+// requests 64 and 47; the gated delta rule 533 and 495, 696 and 660, 89 and 54. What bounds the walk now is its own
+// instructions (the delta rule's: 139 a token and wave, half of them the decays that every block of a head's columns forms).
+template <typename T> struct Four;
+template <> struct Four<float> { typedef float type __attribute__((ext_vector_type(4))); };
+template <> struct Four<bf16> { typedef uint16_t type __attribute__((ext_vector_type(4))); };
+__device__ __forceinline__ float raw_f32(float v) { return v; }
+__device__ __forceinline__ float raw_f32(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
+
+// Where value n of a token's row lies in LDS: fours of values, those that the NS lanes of a column read together side by side.
+// (In plain order the lanes' sixteen bytes lie NPT values apart and meet in half or a quarter of the banks.)
+template <int NS, int NPT> __device__ __forceinline__ int lds_place(int n) { return (n % NPT / 4 * NS + n / NPT) * 4 + n % 4; }
+template <int NS> __device__ __forceinline__ float4 lds_four(const float* row, int ns, int i) {
+    return *reinterpret_cast<const float4*>(row + (i * NS + ns) * 4);
+}
+// The lanes' shares of a token's output, [column][lane], the fours of a column's lanes in an order that changes from one run of
+// 64 shares to the next: the threads that add them up read a column each, sixteen bytes at a time, and would meet in the same banks.
+template <int NS> __device__ __forceinline__ int share_four(int column, int i) {
+    return column * NS + ((i ^ (column / (64 / NS))) & (NS / 4 - 1)) * 4;
+}
+
+template <typename T, int NS, int NPT, bool WIDE> struct StagedRows {
+    static constexpr int NPAD = NS * NPT, W = WIDE ? 4 : 1, PIECES = SCAN_TOKENS * NPAD / W, R = (PIECES + SCAN_THREADS - 1) / SCAN_THREADS;
+    typedef typename Four<T>::type Wide;
+    Wide wide[WIDE ? R : 1];
+    T one[WIDE ? 1 : R];
+    static __device__ __forceinline__ int at(int r) { return ((int)threadIdx.x + r * SCAN_THREADS) * W; }      // the first value's place in the chunk
+    __device__ __forceinline__ void fetch(const T* base, int ld, int N, int c0, int n_tok) {
+        if (WIDE && c0 + SCAN_TOKENS <= n_tok && PIECES >= SCAN_THREADS) {        // a whole chunk: without a condition (beyond N the head's first values, not used)
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int n = at(r) % NPAD;
+                wide[r] = *reinterpret_cast<const Wide*>(base + (size_t)(c0 + at(r) / NPAD) * ld + (n < N ? n : 0));
+            }
+            return;
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int t = c0 + at(r) / NPAD, n = at(r) % NPAD;
+            if (t < n_tok && n < N) {
+                if constexpr (WIDE) wide[r] = *reinterpret_cast<const Wide*>(base + (size_t)t * ld + n);
+                else one[r] = base[(size_t)t * ld + n];
+            }
+        }
+    }
+    // f(r) for the pieces of the chunk's nt tokens (what lies beyond is not walked, and forming it anyway cost a step of single
+    // tokens most: the gated delta rule's 64 requests 93 us against 54). Whole chunks ask no question of their pieces.
+    template <typename F> static __device__ __forceinline__ void each(int nt, F f) {
+        if (nt == SCAN_TOKENS && PIECES % SCAN_THREADS == 0) {
+#pragma unroll
+            for (int r = 0; r < R; r++) f(r);
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                if (at(r) / NPAD < nt) f(r);
+        }
+    }
+    // the values of a live piece, zeros beyond N
+    __device__ __forceinline__ void values(int r, int N, float* f) const {
+        const bool ok = at(r) % NPAD < N;
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            if constexpr (WIDE) f[j] = ok ? raw_f32(wide[r][j]) : 0.f;
+            else f[j] = ok ? to_f32(one[r]) : 0.f;
+        }
+    }
+    static __device__ __forceinline__ void put(int r, float* lds, const float* f) {
+        const int t = at(r) / NPAD, n = at(r) % NPAD;
+        float* to = lds + t * NPAD + lds_place<NS, NPT>(n);
+        if constexpr (WIDE) *reinterpret_cast<float4*>(to) = make_float4(f[0], f[1], f[2], f[3]);
+        else *to = f[0];
+    }
+};
+template <typename T> static bool scan_wide(const void* p, int ld, int N) {
+    return N % 4 == 0 && ld % 4 == 0 && (uintptr_t)p % (4 * sizeof(T)) == 0;
+}
+
+template <typename T, typename TS, int NS, int NPT, bool WIDE>
 __global__ __launch_bounds__(SCAN_THREADS) void linear_scan_kernel(
     const T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk, int heads_per_qk, int N, const T* __restrict__ v,
     int ldv, int P, int gate, const float* __restrict__ decay, const TS* __restrict__ step, int ld_step,
@@ -230,7 +311,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void linear_scan_kernel(
     float* __restrict__ y, int ldy, const TS* __restrict__ step2, const float* __restrict__ step_bias2, float cap, float q_scale,
     float* __restrict__ denom, size_t m_off) {
     constexpr int NPAD = NS * NPT, PT = SCAN_THREADS / NS, TOK = SCAN_TOKENS;
-    constexpr int RK = TOK * NPAD / SCAN_THREADS, RV = (TOK * PT + SCAN_THREADS - 1) / SCAN_THREADS;
+    constexpr int RV = (TOK * PT + SCAN_THREADS - 1) / SCAN_THREADS;
     static_assert(TOK * NPAD % SCAN_THREADS == 0 && NPT % 4 == 0, "the staging loops are whole");
     __shared__ __attribute__((aligned(16))) float k_s[TOK * NPAD];
     __shared__ __attribute__((aligned(16))) float q_s[TOK * NPAD];
@@ -257,39 +338,42 @@ __global__ __launch_bounds__(SCAN_THREADS) void linear_scan_kernel(
     const T* vg = v + (size_t)q0 * ldv + h * P + pz * PT;
     // Two sets of registers take turns: while one chunk of tokens is walked, the loads of the next two are on their way
     // (a trip to memory takes longer than the walk of one chunk).
-    struct Staged { float k[RK], q[RK], v[RV], step, step2; };
+    typedef StagedRows<T, NS, NPT, WIDE> Rows;
+    struct Staged { Rows k, q; T v[RV]; TS step, step2; };
     Staged set_a, set_b;
-    // the tokens c0 .. c0 + TOK - 1 into registers (zeros beyond the request's tokens, beyond N and beyond P)
+    // the tokens c0 .. c0 + TOK - 1 into registers
     auto fetch = [&](Staged& g_, int c0) {
         if (c0 >= n_tok) return;
-#pragma unroll
-        for (int r = 0; r < RK; r++) {
-            const int idx = tid + r * SCAN_THREADS, t = c0 + idx / NPAD, n = idx % NPAD;
-            const bool ok = t < n_tok && n < N;
-            g_.k[r] = ok ? to_f32(kg[(size_t)t * ldk + n]) : 0.f;
-            g_.q[r] = ok ? to_f32(qg[(size_t)t * ldq + n]) : 0.f;
-        }
+        g_.k.fetch(kg, ldk, N, c0, n_tok);
+        g_.q.fetch(qg, ldq, N, c0, n_tok);
 #pragma unroll
         for (int r = 0; r < RV; r++) {
             const int idx = tid + r * SCAN_THREADS, t = c0 + idx / PT, pp = idx % PT;
-            g_.v[r] = (idx < TOK * PT && t < n_tok && pz * PT + pp < P) ? to_f32(vg[(size_t)t * ldv + pp]) : 0.f;
-            if (gate == 2 && idx < TOK * PT && t < n_tok && pz * PT + pp == P) g_.v[r] = 1.f;       // the normaliser's column
+            if (idx < TOK * PT && t < n_tok && pz * PT + pp < P) g_.v[r] = vg[(size_t)t * ldv + pp];
         }
-        g_.step = (gate >= 1 && tid < TOK && c0 + tid < n_tok) ? to_f32(step[(size_t)(q0 + c0 + tid) * ld_step + h]) : 0.f;
-        g_.step2 = (gate == 2 && tid < TOK && c0 + tid < n_tok) ? to_f32(step2[(size_t)(q0 + c0 + tid) * ld_step + h]) : 0.f;
+        if (gate >= 1 && tid < TOK && c0 + tid < n_tok) g_.step = step[(size_t)(q0 + c0 + tid) * ld_step + h];
+        if (gate == 2 && tid < TOK && c0 + tid < n_tok) g_.step2 = step2[(size_t)(q0 + c0 + tid) * ld_step + h];
     };
-    auto stash = [&](const Staged& g_, int c0) {
+    auto stash = [&](const Staged& g_, int c0, int nt) {
+        Rows::each(nt, [&](int r) {
+            float f[Rows::W];
+            g_.k.values(r, N, f);
+            Rows::put(r, k_s, f);
+            g_.q.values(r, N, f);
 #pragma unroll
-        for (int r = 0; r < RK; r++) {
-            k_s[tid + r * SCAN_THREADS] = g_.k[r];
-            q_s[tid + r * SCAN_THREADS] = g_.q[r] * q_scale;
+            for (int j = 0; j < Rows::W; j++) f[j] *= q_scale;
+            Rows::put(r, q_s, f);
+        });
+#pragma unroll
+        for (int r = 0; r < RV; r++) {
+            const int idx = tid + r * SCAN_THREADS, p = pz * PT + idx % PT;
+            if (idx < TOK * PT) v_s[idx] = p < P ? to_f32(g_.v[r]) : p == P && gate == 2 ? 1.f : 0.f;       // 1: the normaliser's column
         }
-#pragma unroll
-        for (int r = 0; r < RV; r++)
-            if (tid + r * SCAN_THREADS < TOK * PT) v_s[tid + r * SCAN_THREADS] = g_.v[r];
+        const bool mine = tid < TOK && c0 + tid < n_tok;
+        const float z1 = gate >= 1 && mine ? to_f32(g_.step) : 0.f, z2 = gate == 2 && mine ? to_f32(g_.step2) : 0.f;
         if (gate == 2) {
             if (tid < WAVE) {                                   // the maximum runs from token to token: one wave, in order
-                const float li = cap * tanhf((g_.step + sb) * inv_cap), zf = cap * tanhf((g_.step2 + sb2) * inv_cap);
+                const float li = cap * tanhf((z1 + sb) * inv_cap), zf = cap * tanhf((z2 + sb2) * inv_cap);
                 const float lf = -(fmaxf(-zf, 0.f) + log1pf(expf(-fabsf(zf))));          // logsigmoid
                 // only the maximum itself is a chain (an add and a maximum a token, the gates read from their lanes); the
                 // exponentials wait until every lane knows its token's maximum and the one before
@@ -313,7 +397,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void linear_scan_kernel(
             }
         } else if (tid < TOK) {
             if (gate == 1) {
-                const float z = g_.step + sb;
+                const float z = z1 + sb;
                 const float dt = fmaxf(z, 0.f) + log1pf(expf(-fabsf(z)));          // softplus, exact for every z
                 a_s[tid] = expf(neg_rate * dt);
                 b_s[tid] = dt;
@@ -326,19 +410,17 @@ __global__ __launch_bounds__(SCAN_THREADS) void linear_scan_kernel(
     auto chunk = [&](Staged& g_, int c0) {
         const int nt = n_tok - c0 < TOK ? n_tok - c0 : TOK;
         __syncthreads();                                   // the walk before has read what is overwritten now
-        stash(g_, c0);
+        stash(g_, c0, nt);
         __syncthreads();
         fetch(g_, c0 + 2 * TOK);
         // A token's operands leave LDS two tokens before (three gained nothing) its multiply-adds: the only chain from token to token is the
         // state's own, and a wave that has a SIMD to itself would otherwise wait for every read.
         struct Operands { float4 k[NPT / 4], q[NPT / 4]; float a, bv; };
         auto read = [&](int t, Operands& o) {
-            const float4* kt = reinterpret_cast<const float4*>(k_s + t * NPAD + ns * NPT);
-            const float4* qt = reinterpret_cast<const float4*>(q_s + t * NPAD + ns * NPT);
 #pragma unroll
             for (int i = 0; i < NPT / 4; i++) {
-                o.k[i] = kt[i];
-                o.q[i] = qt[i];
+                o.k[i] = lds_four<NS>(k_s + t * NPAD, ns, i);
+                o.q[i] = lds_four<NS>(q_s + t * NPAD, ns, i);
             }
             o.a = a_s[t];
             o.bv = b_s[t] * v_s[t * PT + pl];
@@ -357,7 +439,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void linear_scan_kernel(
                 acc0 = fmaf(st[4 * i + 2], qq.z, acc0);
                 acc1 = fmaf(st[4 * i + 3], qq.w, acc1);
             }
-            part_s[t * SCAN_THREADS + tid] = acc0 + acc1;
+            part_s[t * SCAN_THREADS + share_four<NS>(pl, ns / 4) + ns % 4] = acc0 + acc1;
         };
         if (nt == TOK) {
             Operands ring[3];
@@ -380,11 +462,10 @@ __global__ __launch_bounds__(SCAN_THREADS) void linear_scan_kernel(
         for (int idx = tid; idx < nt * PT; idx += SCAN_THREADS) {
             const int t = idx / PT, pp = idx % PT;
             if (pz * PT + pp > P || (pz * PT + pp == P && gate != 2)) continue;
-            const float4* sh = reinterpret_cast<const float4*>(part_s + t * SCAN_THREADS + pp * NS);
             float acc = 0.f;
 #pragma unroll
             for (int i = 0; i < NS / 4; i++) {
-                const float4 u = sh[i];
+                const float4 u = *reinterpret_cast<const float4*>(part_s + t * SCAN_THREADS + share_four<NS>(pp, i));
                 acc = ((acc + u.x) + u.y) + u.z + u.w;
             }
             if (pz * PT + pp == P)
@@ -439,8 +520,15 @@ extern "C" int hfa_linear_scan(const void* q, int ldq, const void* k, int ldk, i
     const size_t m_off = hfa_linear_scan_state_floats(n_heads, qk_dim, v_dim + 1);
     HFA_REQUIRE(n_heads <= 65535 && n_seqs <= 65535 && p_tiles <= 65535, "linear_scan: the step exceeds the grid");
     dim3 grid(n_heads, n_seqs, p_tiles);
+    const bool wide = dtype == HFA_F32 ? scan_wide<float>(q, ldq, qk_dim) && scan_wide<float>(k, ldk, qk_dim)
+                                       : scan_wide<bf16>(q, ldq, qk_dim) && scan_wide<bf16>(k, ldk, qk_dim);
 #define SCAN_GO(T, TS, NS, NPT)                                                                                          \
-    linear_scan_kernel<T, TS, NS, NPT><<<grid, SCAN_THREADS, 0, stream>>>(                                               \
+    do {                                                                                                                 \
+        if (wide) SCAN_AS(T, TS, NS, NPT, true);                                                                         \
+        else SCAN_AS(T, TS, NS, NPT, false);                                                                             \
+    } while (0)
+#define SCAN_AS(T, TS, NS, NPT, WIDE)                                                                                    \
+    linear_scan_kernel<T, TS, NS, NPT, WIDE><<<grid, SCAN_THREADS, 0, stream>>>(                                         \
         (const T*)q, ldq, (const T*)k, ldk, n_heads / qk_heads, qk_dim, (const T*)v, ldv, v_dim, gate, decay, (const TS*)step, \
         ld_step, step_bias, a_log, skip, state, state_ld, q_start, seq_slot, y, ldy, (const TS*)step2, step_bias2, cap, q_scale, \
         denom, m_off)
@@ -457,6 +545,7 @@ extern "C" int hfa_linear_scan(const void* q, int ldq, const void* k, int ldk, i
     else { if (step_dtype == HFA_F32 && gate >= 1) SCAN_SIZES(bf16, float); else SCAN_SIZES(bf16, bf16); }
 #undef SCAN_SIZES
 #undef SCAN_GO
+#undef SCAN_AS
     HFA_LAUNCH_CHECK("linear_scan");
     return 0;
 }
@@ -493,14 +582,14 @@ __device__ __forceinline__ float run_sum(float x) {
 
 // AHEAD: the walk of whole chunks reads operands ahead (steps with prompt portions); without it the kernel needs fewer
 // registers and more blocks share a compute unit, which is what a step of single tokens lives on.
-template <int NS, int NPT, bool AHEAD>
+template <int NS, int NPT, bool AHEAD, bool WIDE>
 __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, int heads_per_qk, int N, const float* __restrict__ v,
     int ldv, int P, const float* __restrict__ a, int lda, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
     const float* __restrict__ b, int ldb, float q_scale, float unit_eps, float* __restrict__ state, size_t state_ld,
     const int* __restrict__ q_start, const int* __restrict__ seq_slot, float* __restrict__ y, int ldy) {
     constexpr int NPAD = NS * NPT, PT = SCAN_THREADS / NS, TOK = SCAN_TOKENS;
-    constexpr int RK = TOK * NPAD / SCAN_THREADS, RV = (TOK * PT + SCAN_THREADS - 1) / SCAN_THREADS;
+    constexpr int RV = (TOK * PT + SCAN_THREADS - 1) / SCAN_THREADS;
     static_assert(TOK * NPAD % SCAN_THREADS == 0 && NPT % 4 == 0, "the staging loops are whole");
     __shared__ __attribute__((aligned(16))) float k_s[TOK * NPAD];
     __shared__ __attribute__((aligned(16))) float q_s[TOK * NPAD];
@@ -522,24 +611,20 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
     const float* qg = q + (size_t)q0 * ldq + g * N;
     const float* ag = a + (size_t)q0 * lda + h * N;
     const float* vg = v + (size_t)q0 * ldv + h * P + pz * PT;
-    float bias_r[RK];                                      // the decay's bias of the channels this thread stages
+    typedef StagedRows<float, NS, NPT, WIDE> Rows;
+    float bias_r[Rows::R * Rows::W];                       // the decay's bias of the channels this thread stages
 #pragma unroll
-    for (int r = 0; r < RK; r++) {
-        const int n = (tid + r * SCAN_THREADS) % NPAD;
+    for (int r = 0; r < Rows::R * Rows::W; r++) {
+        const int n = (Rows::at(r / Rows::W) + r % Rows::W) % NPAD;
         bias_r[r] = n < N ? dt_bias[h * N + n] : 0.f;
     }
-    struct Staged { float k[RK], q[RK], a[RK], v[RV], b; };
+    struct Staged { Rows k, q, a; float v[RV], b; };
     Staged set_a, set_b;
     auto fetch = [&](Staged& g_, int c0) {
         if (c0 >= n_tok) return;
-#pragma unroll
-        for (int r = 0; r < RK; r++) {
-            const int idx = tid + r * SCAN_THREADS, t = c0 + idx / NPAD, n = idx % NPAD;
-            const bool ok = t < n_tok && n < N;
-            g_.k[r] = ok ? kg[(size_t)t * ldk + n] : 0.f;
-            g_.q[r] = ok ? qg[(size_t)t * ldq + n] : 0.f;
-            g_.a[r] = ok ? ag[(size_t)t * lda + n] : 0.f;
-        }
+        g_.k.fetch(kg, ldk, N, c0, n_tok);
+        g_.q.fetch(qg, ldq, N, c0, n_tok);
+        g_.a.fetch(ag, lda, N, c0, n_tok);
 #pragma unroll
         for (int r = 0; r < RV; r++) {
             const int idx = tid + r * SCAN_THREADS, t = c0 + idx / PT, pp = idx % PT;
@@ -547,23 +632,29 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
         }
         g_.b = (tid < TOK && c0 + tid < n_tok) ? b[(size_t)(q0 + c0 + tid) * ldb + h] : 0.f;
     };
-    auto stash = [&](const Staged& g_) {
+    auto stash = [&](const Staged& g_, int nt) {
+        Rows::each(nt, [&](int r) {
+            float f[Rows::W];
+            g_.k.values(r, N, f);
+            Rows::put(r, k_s, f);
+            g_.q.values(r, N, f);
+            Rows::put(r, q_s, f);
+            g_.a.values(r, N, f);
 #pragma unroll
-        for (int r = 0; r < RK; r++) {
-            const int idx = tid + r * SCAN_THREADS;
-            k_s[idx] = g_.k[r];
-            q_s[idx] = g_.q[r];
-            const float z = g_.a[r] + bias_r[r];
-            const float sp = fmaxf(z, 0.f) + log1pf(expf(-fabsf(z)));                 // softplus, exact for every z
-            g_s[idx] = expf(neg_rate * sp);
-        }
+            for (int j = 0; j < Rows::W; j++) {
+                const float z = f[j] + bias_r[r * Rows::W + j];
+                const float sp = fmaxf(z, 0.f) + log1pf(expf(-fabsf(z)));             // softplus, exact for every z
+                f[j] = expf(neg_rate * sp);
+            }
+            Rows::put(r, g_s, f);
+        });
 #pragma unroll
         for (int r = 0; r < RV; r++)
             if (tid + r * SCAN_THREADS < TOK * PT) v_s[tid + r * SCAN_THREADS] = g_.v[r];
         if (tid < TOK) b_s[tid] = 1.0f / (1.0f + expf(-g_.b));
         __syncthreads();
         // unit vectors: a wave a token, the sums of squares in lane order then across the wave
-        for (int t = wv; t < TOK; t += SCAN_THREADS / WAVE) {
+        for (int t = wv; t < nt; t += SCAN_THREADS / WAVE) {
             float sk = 0.f, sq = 0.f;
             for (int n = lane; n < NPAD; n += WAVE) {
                 const float kv = k_s[t * NPAD + n], qv = q_s[t * NPAD + n];
@@ -580,21 +671,18 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
     auto chunk = [&](Staged& g_, int c0) {
         const int nt = n_tok - c0 < TOK ? n_tok - c0 : TOK;
         __syncthreads();                                   // the walk before has read what is overwritten now
-        stash(g_);
+        stash(g_, nt);
         __syncthreads();
         fetch(g_, c0 + 2 * TOK);
         // A token's operands leave LDS two tokens before its multiply-adds (as in linear_scan_kernel): what is left between
         // one token's state and the next is the decay, the sum over the column's lanes, the correction and the write.
         struct Operands { float4 k[NPT / 4], q[NPT / 4], g[NPT / 4]; float beta, v; };
         auto read = [&](int t, Operands& o) {
-            const float4* kt = reinterpret_cast<const float4*>(k_s + t * NPAD + ns * NPT);
-            const float4* qt = reinterpret_cast<const float4*>(q_s + t * NPAD + ns * NPT);
-            const float4* gt = reinterpret_cast<const float4*>(g_s + t * NPAD + ns * NPT);
 #pragma unroll
             for (int i = 0; i < NPT / 4; i++) {
-                o.k[i] = kt[i];
-                o.q[i] = qt[i];
-                o.g[i] = gt[i];
+                o.k[i] = lds_four<NS>(k_s + t * NPAD, ns, i);
+                o.q[i] = lds_four<NS>(q_s + t * NPAD, ns, i);
+                o.g[i] = lds_four<NS>(g_s + t * NPAD, ns, i);
             }
             o.beta = b_s[t];
             o.v = v_s[t * PT + pl];
@@ -628,7 +716,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
                 acc0 = fmaf(st[4 * i + 2], qq.z, acc0);
                 acc1 = fmaf(st[4 * i + 3], qq.w, acc1);
             }
-            part_s[t * SCAN_THREADS + tid] = acc0 + acc1;
+            part_s[t * SCAN_THREADS + share_four<NS>(pl, ns / 4) + ns % 4] = acc0 + acc1;
         };
         if (AHEAD && nt == TOK) {
             Operands ring[3];
@@ -650,11 +738,10 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
         for (int idx = tid; idx < nt * PT; idx += SCAN_THREADS) {
             const int t = idx / PT, pp = idx % PT;
             if (pz * PT + pp >= P) continue;
-            const float4* sh = reinterpret_cast<const float4*>(part_s + t * SCAN_THREADS + pp * NS);
             float acc = 0.f;
 #pragma unroll
             for (int i = 0; i < NS / 4; i++) {
-                const float4 w4 = sh[i];
+                const float4 w4 = *reinterpret_cast<const float4*>(part_s + t * SCAN_THREADS + share_four<NS>(pp, i));
                 acc = ((acc + w4.x) + w4.y) + w4.z + w4.w;
             }
             y[(size_t)(q0 + c0 + t) * ldy + h * P + pz * PT + pp] = acc;
@@ -687,11 +774,14 @@ extern "C" int hfa_delta_scan(const float* q, int ldq, const float* k, int ldk, 
     HFA_REQUIRE(n_heads <= 65535 && n_seqs <= 65535 && p_tiles <= 65535, "delta_scan: the step exceeds the grid");
     dim3 grid(n_heads, n_seqs, p_tiles);
     const bool ahead = max_q_len >= SCAN_TOKENS;            // some request brings a whole chunk
+    const bool wide = scan_wide<float>(q, ldq, qk_dim) && scan_wide<float>(k, ldk, qk_dim) && scan_wide<float>(a, lda, qk_dim);
 #define DELTA_ARGS q, ldq, k, ldk, n_heads / qk_heads, qk_dim, v, ldv, v_dim, a, lda, dt_bias, a_log, b, ldb, q_scale, unit_eps, state, state_ld, q_start, seq_slot, y, ldy
 #define DELTA_GO(NS, NPT)                                                                              \
     do {                                                                                               \
-        if (ahead) delta_scan_kernel<NS, NPT, true><<<grid, SCAN_THREADS, 0, stream>>>(DELTA_ARGS);   \
-        else delta_scan_kernel<NS, NPT, false><<<grid, SCAN_THREADS, 0, stream>>>(DELTA_ARGS);        \
+        if (ahead && wide) delta_scan_kernel<NS, NPT, true, true><<<grid, SCAN_THREADS, 0, stream>>>(DELTA_ARGS);    \
+        else if (ahead) delta_scan_kernel<NS, NPT, true, false><<<grid, SCAN_THREADS, 0, stream>>>(DELTA_ARGS);      \
+        else if (wide) delta_scan_kernel<NS, NPT, false, true><<<grid, SCAN_THREADS, 0, stream>>>(DELTA_ARGS);       \
+        else delta_scan_kernel<NS, NPT, false, false><<<grid, SCAN_THREADS, 0, stream>>>(DELTA_ARGS);                \
     } while (0)
     if (ns == 4) DELTA_GO(4, 4);
     else if (ns == 8 && npt == 4) DELTA_GO(8, 4);
@@ -712,13 +802,13 @@ extern "C" int hfa_delta_scan(const float* q, int ldq, const float* k, int ldk, 
 // what is written; no keys are read); else keys are read. q_act HFA_ACT_SILU: the queries pass silu on their way in. The block,
 // its lanes and the staging through LDS are linear_scan_kernel's, with the decays staged beside the keys as delta_scan_kernel
 // stages its own; nothing crosses lanes inside the walk.
-template <typename T, int NS, int NPT>
+template <typename T, int NS, int NPT, bool WIDE>
 __global__ __launch_bounds__(SCAN_THREADS) void channel_scan_kernel(
     const T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk, int N, const T* __restrict__ v, int ldv, int P,
     const float* __restrict__ decay, int ld_decay, int kcomp, int q_act, float q_scale, float* __restrict__ state, size_t state_ld, const int* __restrict__ q_start,
     const int* __restrict__ seq_slot, float* __restrict__ y, int ldy) {
     constexpr int NPAD = NS * NPT, PT = SCAN_THREADS / NS, TOK = SCAN_TOKENS;
-    constexpr int RK = TOK * NPAD / SCAN_THREADS, RV = (TOK * PT + SCAN_THREADS - 1) / SCAN_THREADS;
+    constexpr int RV = (TOK * PT + SCAN_THREADS - 1) / SCAN_THREADS;
     static_assert(TOK * NPAD % SCAN_THREADS == 0 && NPT % 4 == 0, "the staging loops are whole");
     __shared__ __attribute__((aligned(16))) float k_s[TOK * NPAD];
     __shared__ __attribute__((aligned(16))) float q_s[TOK * NPAD];
@@ -738,55 +828,55 @@ __global__ __launch_bounds__(SCAN_THREADS) void channel_scan_kernel(
     const T* qg = q + (size_t)q0 * ldq + h * N;
     const float* gg = decay + (size_t)q0 * ld_decay + h * N;
     const T* vg = v + (size_t)q0 * ldv + h * P + pz * PT;
-    struct Staged { float k[RK], q[RK], z[RK], v[RV]; };
+    typedef StagedRows<T, NS, NPT, WIDE> Rows;
+    struct Staged { Rows k, q; StagedRows<float, NS, NPT, WIDE> z; T v[RV]; };
     Staged set_a, set_b;
     auto fetch = [&](Staged& g_, int c0) {
         if (c0 >= n_tok) return;
-#pragma unroll
-        for (int r = 0; r < RK; r++) {
-            const int idx = tid + r * SCAN_THREADS, t = c0 + idx / NPAD, n = idx % NPAD;
-            const bool ok = t < n_tok && n < N;
-            g_.k[r] = (ok && !kcomp) ? to_f32(kg[(size_t)t * ldk + n]) : 0.f;
-            g_.q[r] = ok ? to_f32(qg[(size_t)t * ldq + n]) : 0.f;
-            g_.z[r] = ok ? gg[(size_t)t * ld_decay + n] : 0.f;
-        }
+        if (!kcomp) g_.k.fetch(kg, ldk, N, c0, n_tok);
+        g_.q.fetch(qg, ldq, N, c0, n_tok);
+        g_.z.fetch(gg, ld_decay, N, c0, n_tok);
 #pragma unroll
         for (int r = 0; r < RV; r++) {
             const int idx = tid + r * SCAN_THREADS, t = c0 + idx / PT, pp = idx % PT;
-            g_.v[r] = (idx < TOK * PT && t < n_tok && pz * PT + pp < P) ? to_f32(vg[(size_t)t * ldv + pp]) : 0.f;
+            if (idx < TOK * PT && t < n_tok && pz * PT + pp < P) g_.v[r] = vg[(size_t)t * ldv + pp];
         }
     };
-    auto stash = [&](const Staged& g_) {
+    auto stash = [&](const Staged& g_, int nt) {
+        Rows::each(nt, [&](int r) {      // (rows beyond N stay zero)
+            float a[Rows::W], f[Rows::W];
+            const bool live = Rows::at(r) % NPAD < N;
+            g_.z.values(r, N, a);
+            Rows::put(r, g_s, a);
+            if (!kcomp) g_.k.values(r, N, f);
+            else
 #pragma unroll
-        for (int r = 0; r < RK; r++) {
-            const int idx = tid + r * SCAN_THREADS, n = idx % NPAD;
-            const float a = g_.z[r], kk = kcomp ? 1.0f - a : g_.k[r];
-            const bool live = n < N;                       // rows beyond N stay zero
-            g_s[idx] = live ? a : 0.f;
-            k_s[idx] = live ? kk : 0.f;
-            const float qv = g_.q[r];
-            q_s[idx] = (q_act == HFA_ACT_SILU ? qv / (1.0f + expf(-qv)) : qv) * q_scale;
+                for (int j = 0; j < Rows::W; j++) f[j] = live ? 1.0f - a[j] : 0.f;
+            Rows::put(r, k_s, f);
+            g_.q.values(r, N, f);
+#pragma unroll
+            for (int j = 0; j < Rows::W; j++) f[j] = (q_act == HFA_ACT_SILU ? f[j] / (1.0f + expf(-f[j])) : f[j]) * q_scale;
+            Rows::put(r, q_s, f);
+        });
+#pragma unroll
+        for (int r = 0; r < RV; r++) {
+            const int idx = tid + r * SCAN_THREADS;
+            if (idx < TOK * PT) v_s[idx] = pz * PT + idx % PT < P ? to_f32(g_.v[r]) : 0.f;
         }
-#pragma unroll
-        for (int r = 0; r < RV; r++)
-            if (tid + r * SCAN_THREADS < TOK * PT) v_s[tid + r * SCAN_THREADS] = g_.v[r];
     };
     auto chunk = [&](Staged& g_, int c0) {
         const int nt = n_tok - c0 < TOK ? n_tok - c0 : TOK;
         __syncthreads();                                   // the walk before has read what is overwritten now
-        stash(g_);
+        stash(g_, nt);
         __syncthreads();
         fetch(g_, c0 + 2 * TOK);
         struct Operands { float4 k[NPT / 4], q[NPT / 4], g[NPT / 4]; float v; };
         auto read = [&](int t, Operands& o) {
-            const float4* kt = reinterpret_cast<const float4*>(k_s + t * NPAD + ns * NPT);
-            const float4* qt = reinterpret_cast<const float4*>(q_s + t * NPAD + ns * NPT);
-            const float4* gt = reinterpret_cast<const float4*>(g_s + t * NPAD + ns * NPT);
 #pragma unroll
             for (int i = 0; i < NPT / 4; i++) {
-                o.k[i] = kt[i];
-                o.q[i] = qt[i];
-                o.g[i] = gt[i];
+                o.k[i] = lds_four<NS>(k_s + t * NPAD, ns, i);
+                o.q[i] = lds_four<NS>(q_s + t * NPAD, ns, i);
+                o.g[i] = lds_four<NS>(g_s + t * NPAD, ns, i);
             }
             o.v = v_s[t * PT + pl];
         };
@@ -804,7 +894,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void channel_scan_kernel(
                 acc0 = fmaf(st[4 * i + 2], qq.z, acc0);
                 acc1 = fmaf(st[4 * i + 3], qq.w, acc1);
             }
-            part_s[t * SCAN_THREADS + tid] = acc0 + acc1;
+            part_s[t * SCAN_THREADS + share_four<NS>(pl, ns / 4) + ns % 4] = acc0 + acc1;
         };
         if (nt == TOK) {
             Operands ring[3];
@@ -826,11 +916,10 @@ __global__ __launch_bounds__(SCAN_THREADS) void channel_scan_kernel(
         for (int idx = tid; idx < nt * PT; idx += SCAN_THREADS) {
             const int t = idx / PT, pp = idx % PT;
             if (pz * PT + pp >= P) continue;
-            const float4* sh = reinterpret_cast<const float4*>(part_s + t * SCAN_THREADS + pp * NS);
             float acc = 0.f;
 #pragma unroll
             for (int i = 0; i < NS / 4; i++) {
-                const float4 w4 = sh[i];
+                const float4 w4 = *reinterpret_cast<const float4*>(part_s + t * SCAN_THREADS + share_four<NS>(pp, i));
                 acc = ((acc + w4.x) + w4.y) + w4.z + w4.w;
             }
             y[(size_t)(q0 + c0 + t) * ldy + h * P + pz * PT + pp] = acc;
@@ -896,10 +985,18 @@ extern "C" int hfa_channel_scan(const void* q, int ldq, const void* k, int ldk, 
     const int pt = SCAN_THREADS / ns, p_tiles = (v_dim + pt - 1) / pt;
     HFA_REQUIRE(n_heads <= 65535 && n_seqs <= 65535 && p_tiles <= 65535, "channel_scan: the step exceeds the grid");
     dim3 grid(n_heads, n_seqs, p_tiles);
-#define CH_GO(T, NS, NPT)                                                                                                      \
-    channel_scan_kernel<T, NS, NPT><<<grid, SCAN_THREADS, 0, stream>>>((const T*)q, ldq, (const T*)k, ldk, qk_dim, (const T*)v, ldv, v_dim, \
-                                                                       decay, ld_decay, kcomp, q_act, q_scale, state, state_ld, q_start,  \
-                                                                       seq_slot, y, ldy)
+    const bool wide = scan_wide<float>(decay, ld_decay, qk_dim) && (dtype == HFA_F32
+        ? scan_wide<float>(q, ldq, qk_dim) && (kcomp || scan_wide<float>(k, ldk, qk_dim))
+        : scan_wide<bf16>(q, ldq, qk_dim) && (kcomp || scan_wide<bf16>(k, ldk, qk_dim)));
+#define CH_AS(T, NS, NPT, WIDE)                                                                                                \
+    channel_scan_kernel<T, NS, NPT, WIDE><<<grid, SCAN_THREADS, 0, stream>>>((const T*)q, ldq, (const T*)k, ldk, qk_dim, (const T*)v, \
+                                                                             ldv, v_dim, decay, ld_decay, kcomp, q_act, q_scale, state, \
+                                                                             state_ld, q_start, seq_slot, y, ldy)
+#define CH_GO(T, NS, NPT)                      \
+    do {                                       \
+        if (wide) CH_AS(T, NS, NPT, true);     \
+        else CH_AS(T, NS, NPT, false);         \
+    } while (0)
 #define CH_SIZES(T)                                          \
     do {                                                     \
         if (ns == 4) CH_GO(T, 4, 4);                         \
@@ -913,6 +1010,7 @@ extern "C" int hfa_channel_scan(const void* q, int ldq, const void* k, int ldk, 
     else CH_SIZES(bf16);
 #undef CH_SIZES
 #undef CH_GO
+#undef CH_AS
     HFA_LAUNCH_CHECK("channel_scan");
     return 0;
 }
