@@ -22,11 +22,11 @@
 //   M in 33 .. 128   gemm_stream_kernel (gemm_stream.hip) if N is a multiple of 128 and K of 64, the output
 //                    has fewer than 512 tiles and a block gets 16 units or more; else gemm_mfma_kernel
 //                    with tiles of 64 x 128 or 128 x 128
-//   M > 64           gemm_dma_kernel (below) with tiles of 256 rows, if M wastes few of them and the
-//                    output has 128 tiles of 256 x 256 (tiles of 256 x 192 where those need fewer rounds
-//                    over the CUs; with fewer K is cut into parts that give every CU a block, with tiles of
-//                    256 x 128 if M is at most 256; or the tiles are 256 x 128 without parts); else
-//                    gemm_mfma_kernel with tiles of 128 x 128
+//   M in 65 .. 128   gemm_dma_kernel (below) with tiles of 256 rows where M wastes few of them, else gemm_mfma_kernel with
+//                    tiles of 128 x 128
+//   M > 128          the tiles (256 x 256, 256 x 192, 256 x 128 or 128 x 128 of gemm_dma_kernel, 128 x 128 of
+//                    gemm_mfma_kernel) and the parts of K by rows wasted and rounds over the CUs, unless a formula fitted to
+//                    measured times gives others 6 % less (better_tiles)
 #include <type_traits>
 
 #include "common.h"
